@@ -27,9 +27,11 @@
 #if defined(__HIPCC__)
 #define BX_POW_TABLE static __device__ __constant__ const
 #define BX_POW_FN __device__ __forceinline__
+#define BX_POW_MEMBER __device__ __forceinline__
 #else
 #define BX_POW_TABLE static const
 #define BX_POW_FN static inline
+#define BX_POW_MEMBER inline // of a struct: a static member function takes no const
 #endif
 
 #include "bx_pow_tables.h"
@@ -311,10 +313,10 @@ BX_POW_FN void ddu_powi(double x, int n, double &h, double &l)
 // the same values (a kernel's copy in LDS).
 struct ConstTables
 {
-    BX_POW_FN double invc(int j) const { return bx_log_invc[j]; }
-    BX_POW_FN double logc(int j) const { return bx_log_logc_hi[j]; }
-    BX_POW_FN double r7c(int j) const { return bx_r7_invc[j]; }
-    BX_POW_FN double r7two(int i) const { return bx_r7_two[i]; }
+    BX_POW_MEMBER double invc(int j) const { return bx_log_invc[j]; }
+    BX_POW_MEMBER double logc(int j) const { return bx_log_logc_hi[j]; }
+    BX_POW_MEMBER double r7c(int j) const { return bx_r7_invc[j]; }
+    BX_POW_MEMBER double r7two(int i) const { return bx_r7_two[i]; }
 };
 
 // log(x) to ~1e-11 absolute, x positive and normal (same table split as

@@ -21,8 +21,7 @@ D = ctypes.POINTER(ctypes.c_double)
 def lib():
     global _lib
     if _lib is None:
-        if not os.path.exists(PATH):
-            subprocess.run(["make", "-s", "-C", HERE], check=True)
+        subprocess.run(["make", "-s", "-C", HERE], check=True)
         _lib = ctypes.CDLL(PATH)
         _lib.or_helm_apply.argtypes = [ctypes.c_int, ctypes.c_int, D, D, D, D, D, D, D, ctypes.c_double,
                                        ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double, D]

@@ -4,7 +4,8 @@ TEST INFRASTRUCTURE ONLY: imported by tests/, __graft_entry__.smoke() and
 bench.py's cpu_baseline leg, as the checker / CPU baseline.  The product
 (bamrex_amd) never imports it.
 
-Build with `make -C oracle` (done by __graft_entry__.build()).
+Build with `make -C oracle` (done by __graft_entry__.build()); a library older
+than its sources is built again when it is loaded.
 """
 import ctypes
 import os
@@ -71,8 +72,7 @@ def _load(bxpow):
     if key in _libs:
         return _libs[key]
     path = os.path.join(BUILD, "liboracle_bxpow.so" if bxpow else "liboracle.so")
-    if not os.path.exists(path):
-        build()
+    build()
     l = ctypes.CDLL(path)
     for n, a in _SIGS.items():
         getattr(l, n).argtypes = a
