@@ -2029,8 +2029,10 @@ extern "C" int bx_helm_solve(bx_helm *h, const double *b, double *x, int method,
                 return rc;
         }
     }
-    // the last kernel of either solver mailed the final norm: everything
-    // before it has completed
+    // The message that carried the final norm is posted by the launch that
+    // still stores the iterate, and more may follow it: the copy of an iterate
+    // that ended in the other array, kernels of an iteration launched ahead.
+    H_CHECK(hipStreamSynchronize(s));
     st->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0)
                       .count();
     return BX_OK;
