@@ -1289,6 +1289,8 @@ extern "C" int bx_get_tuning(const bx_ctx *c, bx_tuning *out)
     if (!c || !out)
         return set_error(BX_ERR_INVALID, "bx_get_tuning: null argument");
     *out = c->tune;
+    if (c->level_set)
+        out->seg_k = c->seg_k; // the length in use, chosen or set
     return BX_OK;
 }
 

@@ -178,7 +178,8 @@ typedef struct
     int block_t;      /* threads per block of the y/z sweeps */
     int seg_k;        /* cells per lane along y/z; until a shape is set
                        * (bx_set_tuning, bx_autotune) the library chooses the
-                       * length by the level's size instead */
+                       * length by the level's size instead, and
+                       * bx_get_tuning reports the one in use */
     int grid_cap;     /* max resident blocks per CU used for persistent grids */
 } bx_tuning;
 
