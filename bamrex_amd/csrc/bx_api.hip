@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -306,6 +307,9 @@ static long long t_items(const bx_ctx *c, const bx_box &bx, int d, int K)
     return (q + 63) / 64;
 }
 
+// segment lengths of the y/z sweeps to choose from
+constexpr int SEG_KS[] = { 1, 2, 3, 4, 6, 8, 11, 16, 22, 32, 43, 64, 128 };
+
 // Segment length of the y/z sweeps when no shape was set.  A segment of K
 // cells costs its lane K + 1 face fluxes and K + 2 reconstructions, so long
 // segments do the least work; but a level has (cells / K) / 64 segments'
@@ -319,12 +323,11 @@ static long long t_items(const bx_ctx *c, const bx_box &bx, int d, int K)
 // 32 would take 118), 4096^2 505 -> 458 (43).
 static int choose_seg_k(const bx_ctx *c)
 {
-    const int       ks[] = { 1, 2, 3, 4, 6, 8, 11, 16, 22, 32, 43, 64, 128 };
     const int       wpb  = c->tune.block_t / 64;
     double          best = 0;
     int             best_k = 16;
     const long long simds = 4LL * c->ncu;
-    for (int K : ks)
+    for (int K : SEG_KS)
     {
         double t = 0;
         for (int d = 1; d < c->D; ++d)
@@ -1353,12 +1356,31 @@ static int time_sweep(bx_ctx *c, int dir, const double dx[3], double *U,
     return rc;
 }
 
+// All sweeps of the shape in use: ms becomes the smaller of what it was and
+// the time now.
+static int time_shape(bx_ctx *c, const double dx[3], double *U, double *U_tmp, hipStream_t s,
+                      double ms[3])
+{
+    for (int d = 0; d < c->D; ++d)
+    {
+        double t = 0;
+        int    rc;
+        if ((rc = time_sweep(c, d, dx, U, U_tmp, s, 5, &t)) != BX_OK)
+            return rc;
+        ms[d] = std::min(ms[d], t);
+    }
+    return BX_OK;
+}
+
 // The search itself; on an error the caller restores the entry shape.
 static int autotune_search(bx_ctx *c, const double dx[3], double *U, double *U_tmp,
                            hipStream_t s, double *best_ms)
 {
-    int       rc;
-    bx_tuning best = c->tune;
+    int             rc;
+    const bx_tuning entry       = c->tune;
+    const bool      entry_tuned = c->tuned;
+    bx_tuning       best        = entry;
+    best.seg_k                  = c->seg_k; // the length in use
     // untimed sweeps at the entry shape first: after an idle period the GPU
     // clock dips over the first ~10 ms of back-to-back work, which would
     // bias the first candidates
@@ -1368,13 +1390,14 @@ static int autotune_search(bx_ctx *c, const double dx[3], double *U, double *U_t
                 return rc;
     const int blocks[3] = { 64, 128, 256 };
     const int caps[4]   = { 0, 1, 2, 4 };
-    // segment lengths: powers of two, and the median box length along the
-    // transverse sweeps split into m equal parts (m = 1..8), which lets the
-    // item count divide evenly over 2, 3, ... resident waves per SIMD;
+    // segment lengths: those choose_seg_k picks from, and the median box length
+    // along the transverse sweeps split into m equal parts (m = 1..8), which
+    // lets the item count divide evenly over 2, 3, ... resident waves per SIMD;
     // lengths above what bx_set_tuning accepts are skipped
-    std::vector<int> ks = { 8, 16, 32, 64, 128 };
+    std::vector<int> ks;
     if (c->D >= 2)
     {
+        ks.assign(std::begin(SEG_KS), std::end(SEG_KS));
         std::vector<int> len;
         for (const bx_box &bx : c->hboxes)
             len.push_back(bx.hi[1] - bx.lo[1] + 1);
@@ -1431,19 +1454,22 @@ static int autotune_search(bx_ctx *c, const double dx[3], double *U, double *U_t
                 }
             }
     }
-    if ((rc = bx_set_tuning(c, &best)) != BX_OK)
+    // the shape found against the one the level came with, which may be none
+    // of the candidates (and the grid cap is searched with the x sweep alone),
+    // in turn: a difference of a few percent counts here
+    double e_ms[3] = { 1e30, 1e30, 1e30 }, b_ms[3] = { 1e30, 1e30, 1e30 };
+    for (int k = 0; k < 3; ++k)
+        if ((rc = apply_shape(c, entry, entry_tuned)) != BX_OK
+            || (rc = time_shape(c, dx, U, U_tmp, s, e_ms)) != BX_OK
+            || (rc = bx_set_tuning(c, &best)) != BX_OK
+            || (rc = time_shape(c, dx, U, U_tmp, s, b_ms)) != BX_OK)
+            return rc;
+    const bool keep = std::accumulate(e_ms, e_ms + c->D, 0.0)
+                      <= std::accumulate(b_ms, b_ms + c->D, 0.0);
+    if (keep && (rc = apply_shape(c, entry, entry_tuned)) != BX_OK)
         return rc;
-    if (best_ms)
-    {
-        best_ms[0] = bx_ms;
-        for (int d = 1; d < c->D; ++d)
-        {
-            double ms = 0;
-            if ((rc = time_sweep(c, d, dx, U, U_tmp, s, 5, &ms)) != BX_OK)
-                return rc;
-            best_ms[d] = ms;
-        }
-    }
+    for (int d = 0; best_ms && d < c->D; ++d)
+        best_ms[d] = keep ? e_ms[d] : b_ms[d];
     return BX_OK;
 }
 

@@ -187,7 +187,8 @@ int bx_get_tuning(const bx_ctx *ctx, bx_tuning *out);
 int bx_set_tuning(bx_ctx *ctx, const bx_tuning *t);
 
 /* Times every candidate launch shape of every sweep direction on (U, U_tmp)
- * and keeps the fastest (block size x segment length x grid cap).  The state
+ * and keeps the fastest (block size x segment length x grid cap), or the shape
+ * the level came with where no candidate is faster.  The state
  * buffers are overwritten.  Synchronous; writes the timings (ms per sweep)
  * of the winning shapes to best_ms[dir] when best_ms is not NULL. */
 int bx_autotune(bx_ctx *ctx, const double dx[3], double dt, double *U,

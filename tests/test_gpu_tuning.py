@@ -1,4 +1,5 @@
-"""Launch shapes of the sweeps: the one that is reported."""
+"""Launch shapes of the sweeps: the one that is reported, and what a search may
+choose."""
 import pytest
 
 from bamrex_amd.level import Level, make_params
@@ -31,5 +32,17 @@ def test_reported_shape_is_the_one_in_use(n, box):
         assert lev.get_tuning() == dict(t, block_x=128)
         lev.set_tuning(seg_k=24)
         assert lev.get_tuning() == dict(t, block_x=128, seg_k=24)
+    finally:
+        lev.close()
+
+
+def test_autotune_of_a_small_level_finds_short_segments():
+    """256^2 cells: one cell per lane (the length used without a shape) sweeps
+    about 3 times as fast as 8, the shortest length that was searched."""
+    announce("autotune 256^2")
+    lev = level(256, 64)
+    try:
+        lev.autotune([1 / 256, 1 / 256], 1e-4)
+        assert lev.get_tuning()["seg_k"] < 8
     finally:
         lev.close()
