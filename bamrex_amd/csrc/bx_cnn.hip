@@ -749,7 +749,10 @@ __global__ __launch_bounds__(256) void k_train_bwd16(
         }
         if (LAST)
         {
-            // the wave's own rows of sg1 (written by this wave), all taps of x
+            // the wave's own rows of sg1, written by other lanes of this wave:
+            // ordered within the wave, no workgroup barrier; all taps of x
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll 4
             for (int xx = 0; xx < TT; ++xx)
                 a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(
