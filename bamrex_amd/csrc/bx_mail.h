@@ -47,7 +47,10 @@ struct MailBox
         }
         for (int k = 0; k < MAIL_SLOTS; ++k)
             slots[k] = Mail();
-        return hipHostGetDevicePointer((void **)&dev, slots, 0);
+        e = hipHostGetDevicePointer((void **)&dev, slots, 0);
+        if (e != hipSuccess)
+            close(); // open or closed, nothing between: kernels post to dev
+        return e;
     }
     void close()
     {
