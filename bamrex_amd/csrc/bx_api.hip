@@ -230,7 +230,7 @@ extern "C" int bx_create(const bx_params *params, bx_ctx **out)
     if (hipMalloc((void **)&c->d_maxbits, maxbytes) != hipSuccess
         || hipMalloc((void **)&c->d_dt, 64) != hipSuccess
         || hipMalloc((void **)&c->d_time, 64) != hipSuccess
-        || hipMalloc((void **)&c->d_step, 64) != hipSuccess)
+        || hipMalloc((void **)&c->d_last, 64) != hipSuccess)
     {
         bx_destroy(c);
         return set_error(BX_ERR_HIP, "bx_create: hipMalloc failed");
@@ -238,8 +238,7 @@ extern "C" int bx_create(const bx_params *params, bx_ctx **out)
     (void)hipMemset(c->d_maxbits, 0, maxbytes);
     (void)hipMemset(c->d_dt, 0, 64);
     (void)hipMemset(c->d_time, 0, 64);
-    (void)hipMemset(c->d_step, 0, 64);
-    c->d_last = c->d_step + 1;
+    (void)hipMemset(c->d_last, 0, 64);
     *out = c;
     return BX_OK;
 }
@@ -264,7 +263,7 @@ extern "C" void bx_destroy(bx_ctx *c)
     free_dev(c->d_maxbits);
     free_dev(c->d_dt);
     free_dev(c->d_time);
-    free_dev(c->d_step);
+    free_dev(c->d_last);
     c->mail.close(); // hipFree above has waited for the device
     delete c;
 }
@@ -1137,7 +1136,6 @@ static int step_device(bx_ctx *c, long long n, const double dx[3], double cfl, d
         if (d == D - 1)
         {
             t.time_out = c->d_time + (n + 1) % 2;
-            t.step     = c->d_step;
             t.mail     = c->mail.dev;
             t.seq      = seq;
         }
@@ -1211,7 +1209,7 @@ extern "C" int bx_run(bx_ctx *c, const double dx[3], double cfl,
     int         rc;
     if ((rc = do_fill_all(c, U, s)) != BX_OK)
         return rc;
-    BX_HIP_CHECK(launch_run_init(c->d_maxbits, c->d_time, start_time, c->d_step, c->d_last, s));
+    BX_HIP_CHECK(launch_run_init(c->d_maxbits, c->d_time, start_time, c->d_last, s));
     if ((rc = launch_maxspeed(c, U, s)) != BX_OK)
         return rc;
 

@@ -178,7 +178,6 @@ __device__ __forceinline__ double step_begin(const StepCtl &c, const double *d_d
     {
         const double t = *c.time_in + dt;
         *c.time_out    = t;
-        *c.step        = *c.step + 1;
         if (c.gate.last)
         {
             if (c.stop_time >= 0.0 && !(t < c.stop_time))
@@ -742,14 +741,13 @@ __global__ void k_compute_dt(unsigned long long *d_maxbits, double *d_dt,
 }
 
 __global__ void k_run_init(unsigned long long *d_maxbits, double *d_time, double time,
-                           long long *d_step, long long *d_last)
+                           long long *d_last)
 {
     if (threadIdx.x < MAX_SLOTS)
         d_maxbits[threadIdx.x * MAX_SLOT_WORDS] = 0ULL;
     if (threadIdx.x != 0)
         return;
     *d_time = time;
-    *d_step = 0;
     *d_last = 0x7fffffffffffffffLL;
 }
 
@@ -988,10 +986,10 @@ hipError_t launch_compute_dt(unsigned long long *d_maxbits, double *d_dt,
 }
 
 hipError_t launch_run_init(unsigned long long *d_maxbits, double *d_time, double time,
-                           long long *d_step, long long *d_last, hipStream_t stream)
+                           long long *d_last, hipStream_t stream)
 {
     hipLaunchKernelGGL(k_run_init, dim3(1), dim3(64), 0, stream, d_maxbits, d_time, time,
-                       d_step, d_last);
+                       d_last);
     return hipGetLastError();
 }
 

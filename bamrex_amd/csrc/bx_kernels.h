@@ -32,7 +32,6 @@ struct StepCtl
     double                   *dt        = nullptr;
     const double             *time_in   = nullptr;
     double                   *time_out  = nullptr; // last sweep: the new time
-    long long                *step      = nullptr;
     double                    dx[3]     = { 0, 0, 0 };
     double                    cfl       = 0;
     double                    stop_time = -1;
@@ -117,10 +116,10 @@ hipError_t launch_compute_dt(unsigned long long *d_maxbits, double *d_dt,
                              const double *d_time, int D, const double dx[3],
                              double cfl, double stop_time, hipStream_t stream);
 
-// the state of a time loop before its first step: the time, no steps, every
+// the state of a time loop before its first step: the time, no last step, every
 // speed accumulator zero
 hipError_t launch_run_init(unsigned long long *d_maxbits, double *d_time, double time,
-                           long long *d_step, long long *d_last, hipStream_t stream);
+                           long long *d_last, hipStream_t stream);
 
 hipError_t launch_set_u64(unsigned long long *p, unsigned long long v,
                           hipStream_t stream);

@@ -78,7 +78,6 @@ struct bx_ctx
 
     unsigned long long *d_maxbits = nullptr; // MAX_SLOTS accumulators (StepCtl)
     double             *d_dt = nullptr, *d_time = nullptr; // two times
-    long long          *d_step = nullptr;
     long long          *d_last = nullptr; // StepGate
     MailBox             mail;
 
