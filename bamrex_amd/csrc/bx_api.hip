@@ -607,8 +607,11 @@ static void build_ghost_segments(bx_ctx *c)
                         for (int is = 0; is < nb; ++is)
                         {
                             const bx_box &sb = B[is];
-                            int           qlo[3], qhi[3];
-                            bool          ok = true;
+                            // nearly every box, looked at once per piece
+                            if (ihi[0] < sb.lo[0] || ilo[0] > sb.hi[0])
+                                continue;
+                            int  qlo[3], qhi[3];
+                            bool ok = true;
                             for (int d = 0; d < 3 && ok; ++d)
                             {
                                 const int slo = d < D ? sb.lo[d] : 0;
