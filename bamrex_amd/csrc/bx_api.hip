@@ -317,9 +317,9 @@ constexpr int SEG_KS[] = { 1, 2, 3, 4, 6, 8, 11, 16, 22, 32, 43, 64, 128 };
 // segments win while SIMDs are idle.  The estimate of a sweep, in face times of
 // one wave: rounds of resident waves x (K + 1.5) x max(2, waves per SIMD).
 // Measured y sweeps (MI355X, minbee), K = 16 against the length chosen:
-// 256^2 38.8 -> 10.4 us (K = 1), 512^2 39.8 -> 17.8 (2), 1024^2 41.8 -> 37.6
-// (8), 1.44 M cells in uneven boxes 62.5 -> 57.6 (4), 2048^2 162 -> 125 (11;
-// 32 would take 118), 4096^2 505 -> 458 (43).
+// 256^2 34.9 -> 9.7 us (K = 1), 512^2 35.8 -> 15.7 (2), 1024^2 37.5 -> 33.0
+// (8), 1.44 M cells in uneven boxes 60.0 -> 54.4 (4), 2048^2 141 -> 105 (32;
+// 22 would take 102), 4096^2 419 -> 381 (128); 192^3 289 -> 268 (64).
 static int choose_seg_k(const bx_ctx *c)
 {
     const int       wpb  = c->tune.block_t / 64;

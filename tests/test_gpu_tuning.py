@@ -38,7 +38,7 @@ def test_reported_shape_is_the_one_in_use(n, box):
 
 def test_autotune_of_a_small_level_finds_short_segments():
     """256^2 cells: one cell per lane (the length used without a shape) sweeps
-    about 3 times as fast as 8, the shortest length that was searched."""
+    in 9.7 us against 21.4 for 8, once the shortest length that was searched."""
     announce("autotune 256^2")
     lev = level(256, 64)
     try:
